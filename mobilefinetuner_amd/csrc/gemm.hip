@@ -644,7 +644,7 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
   float* wsp = ws.ptr ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws.ptr) + skew) : nullptr;
   const size_t ws_bytes = ws.ptr && ws.bytes > skew ? ws.bytes - skew : 0;
   XPlan pl = plan_gemm_x(M, N, K, k_max, ws_bytes, nm != nullptr && N % 4 == 0 && N <= 4096 && ldc == N,
-                         ep.stats != nullptr, b_f16);
+                         ep.stats != nullptr);
   // Tuning hook: MFT_GEMM_PLAN="bm,bn,splits" (or per shape, "M,N,K:bm,bn,splits;...") forces tiles and a uniform split.
   static const char* forced_env = getenv("MFT_GEMM_PLAN");
   int bm = 0, bn = 0, sp = 0;
@@ -652,6 +652,8 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
       ((bm == 64 && bn == 64) || (bm == 64 && bn == 128) || (bm == 128 && bn == 128)) && sp >= 1 &&
       (sp == 1 || (size_t)sp * M * N * sizeof(float) <= ws_bytes))
     pl = {bm, bn, sp, (int)(cdiv(M, bm) * cdiv(N, bn)), 0};
+  MFT_CHECK_ARG(!ep.stats || (pl.bn == 128 && pl.splits == 1 && pl.tail_splits <= 1),
+                "row statistics need whole 128-wide tiles");
   static const bool log_plans = getenv("MFT_GEMM_PLAN_LOG") != nullptr;  // tuning hook: print each launch's plan
   if (log_plans)
     fprintf(stderr, "gemm %d,%d,%d:%d,%d,%d full=%d tail=%d norm=%d\n", M, N, K, pl.bm, pl.bn, pl.splits, pl.full,

@@ -255,17 +255,17 @@ dim3 xcd_grid(Params& p, int splits) {
 }
 
 // gemm_x.hip.  How gemm_x_launch runs C = A·op(B): tiles bm×bn of 64×64,
-// 64×128 or 128×128 (64×64 with fp16 B); with splits > 1 every tile in that
-// many K-slices to [slice][M][N] partials in ws, which the caller reduces;
-// else the first `full` tiles whole and the others in tail_splits slices,
-// summed by a second launch.
+// 64×128 or 128×128; with splits > 1 every tile in that many K-slices to
+// [slice][M][N] partials in ws, which the caller reduces; else the first
+// `full` tiles whole and the others in tail_splits slices, summed by a second
+// launch.
 struct XPlan {
   int bm, bn, splits, full, tail_splits;
 };
 // norm: a row norm of the finished output follows (it rides in the
 // reduction of a uniform split); stats: 128-wide tiles, none split.
 // k_max: the deepest K-slice a tile may take.
-XPlan plan_gemm_x(int M, int N, int K, int64_t k_max, size_t ws_bytes, bool norm, bool stats, bool b_f16);
+XPlan plan_gemm_x(int M, int N, int K, int64_t k_max, size_t ws_bytes, bool norm, bool stats);
 int gemm_x_depth(const XPlan& pl, const GemmParams& p);  // the deepest K-slice of a plan
 void gemm_x_launch(hipStream_t s, GemmParams& p, const XPlan& pl, bool b_nk, bool b_f16, float* ws,
                    const KernelEvents* tail_ev);

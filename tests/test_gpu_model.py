@@ -65,6 +65,9 @@ SMALL = {
     # first 64-column block is ragged and whose second lies wholly past the
     # vocabulary; two micro-batches offset the statistics rows.
     "qwen2-wide-vocab": (qwen2(1, 128, 2, 1, 64, 256, vocab=70001, name="qwen-wv"), 2, 96, 2),
+    # The same with fp16-stored weights whose width (100) the fp16 matrix-core
+    # kernel does not take: the widened GEMM writes the statistics.
+    "qwen2-fp16w-wide-vocab": (qwen2(1, 100, 2, 1, 64, 256, vocab=70001, name="qwen-wv16", w_fp16=1), 2, 96, 2),
     "gpt2-wide-vocab": (gpt2(1, 128, 2, vocab=53672, max_pos=128, name="gpt2-wv"), 2, 96, 2),
 }
 
