@@ -298,6 +298,37 @@ def test_fp32_linear_values_without_a_split(M, K, N):
     assert np.all(np.abs(y[ok] - ref[ok]) <= (K / 2 + 16) * 2.0 ** -23 * mag[ok])  # an fp32 chain: K/2 additions
 
 
+@pytest.mark.parametrize("same_sign", [False, True])
+@pytest.mark.parametrize("K", [768, 4864])
+def test_fp32_linear_tiny_against_large(K, same_sign):
+    """Operands whose bf16 terms would fall below bf16's normal range, down to
+    the smallest fp32 values, against large ones, in either place: an fp32
+    chain's bound (K/2 + 16 additions, each off by at most 2^-23 of the sum of
+    magnitudes, and by half of 2^-149)."""
+    M, N = 72, 64
+    for xe, we in [(-108, 10), (-112, 20), (-118, 20), (-122, 23), (-122, 40), (-126, 40), (-131, 60), (-140, 100), (-149, 110)]:
+        print(f"tiny against large K={K} x~2^{xe} w~2^{we}", flush=True)
+        a = (np.ldexp(RNG.uniform(1, 2, (M, K)), xe)).astype(np.float32)
+        b = (np.ldexp(RNG.uniform(1, 2, (K, N)), we)).astype(np.float32)
+        if not same_sign:
+            a *= RNG.choice([-1, 1], a.shape).astype(np.float32)
+            b *= RNG.choice([-1, 1], b.shape).astype(np.float32)
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+        bound = (K / 2 + 16) * (2.0 ** -23 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + 2.0 ** -150)
+        y = h(ops.lora_linear_fwd(g(a), g(b), None, None, None, 1.0)[0])
+        assert np.all(np.abs(y - ref) <= bound), (xe, we, np.max(np.abs(y - ref) / bound))
+        yt = h(ops.lora_linear_fwd(g(b.T.copy()), g(a.T.copy()), None, None, None, 1.0)[0])
+        assert np.all(np.abs(yt.T - ref) <= bound), (we, xe, np.max(np.abs(yt.T - ref) / bound))
+        dx = h(ops.lora_linear_bwd(g(a), None, g(b.T.copy()), None, None, None, 1.0)[0])
+        assert np.all(np.abs(dx - ref) <= bound), (xe, we, np.max(np.abs(dx - ref) / bound))
+        # fp16 W at a depth the fp16 kernel does not take
+        a16, w16 = a[:, :K - 4], np.ldexp(b[:K - 4], min(we, 14) - we).astype(np.float16)
+        ref16 = a16.astype(np.float64) @ w16.astype(np.float64)
+        b16 = (K / 2 + 16) * (2.0 ** -23 * (np.abs(a16).astype(np.float64) @ np.abs(w16).astype(np.float64)) + 2.0 ** -150)
+        y16 = h(ops.lora_linear_fwd(g(a16), g(w16), None, None, None, 1.0)[0])
+        assert np.all(np.abs(y16 - ref16) <= b16), (xe, we, np.max(np.abs(y16 - ref16) / b16))
+
+
 @pytest.mark.parametrize("M,K,r", [(1, 8, 32), (511, 2048, 8), (513, 2052, 4), (1025, 2048, 8), (1027, 2300, 4),
                                    (70, 2048, 16), (33, 516, 32)])
 def test_rank_projection_row_groups(M, K, r):
