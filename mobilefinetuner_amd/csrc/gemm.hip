@@ -635,9 +635,10 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
                               !ep.gelu_grad_of && !ep.P && !(ep.norm && ep.norm->kind != NORM_NONE)),
                 "row statistics describe plain logits (no epilogue terms)");
   // a tile's K-slice is addressed through 32-bit buffer offsets from the
-  // tile's first row / column: the deepest slice they reach
+  // tile's first row / column: the deepest slice they reach in both operands
   const int64_t reach = (int64_t(1) << 32) / (b_f16 ? 2 : 4) - 1;
-  const int64_t k_max = b_nk ? reach - 128 * p.ldb : (reach - 128) / p.ldb;
+  const int64_t k_max =
+      std::min((int64_t(1) << 30) - 1 - 128 * lda, b_nk ? reach - 128 * p.ldb : (reach - 128) / p.ldb);
 
   const RowNorm* nm = ep.norm && ep.norm->kind != NORM_NONE ? ep.norm : nullptr;
   const size_t skew = ws.ptr ? (16 - ((uintptr_t)ws.ptr & 15)) & 15 : 0;  // partials are moved 16 bytes at a time
@@ -672,8 +673,7 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
     tev.stop = ev->tail_stop;
   }
   t_gemm_events = dispatch_events ? ev : nullptr;
-  MFT_CHECK_ARG((int64_t)128 * lda + K < (int64_t(1) << 30) && gemm_x_depth(pl, p) <= k_max,
-                "GEMM operand too large for 32-bit buffer offsets");
+  MFT_CHECK_ARG(gemm_x_depth(pl, p) <= k_max, "GEMM operand too large for 32-bit buffer offsets");
   gemm_x_launch(s, p, pl, b_nk, b_f16, wsp, tev.start ? &tev : nullptr);
   t_gemm_events = nullptr;
   if (ev && ev->stop && !dispatch_events) MFT_HIP(hipEventRecord(ev->stop, s));

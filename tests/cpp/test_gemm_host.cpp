@@ -1,0 +1,66 @@
+// test_gemm_host.cpp — host side of the fp32 GEMMs, without a GPU: what
+// gemm() refuses and accepts.  An accepted call gets as far as its launch,
+// which fails here for want of a device (MFT_EHIP); a refused one throws
+// MFT_EINVAL before.  The operands are addresses that nothing reads.
+#include <cstdio>
+#include <cstring>
+
+#include "gemm_common.h"
+
+using namespace mft;
+
+namespace {
+
+float* at(uintptr_t a) { return reinterpret_cast<float*>(a); }
+
+int status_of(int M, int N, int K, bool b_nk, int64_t lda, int64_t ldb, size_t ws_bytes, const KernelEvents* ev = nullptr) {
+  Scratch ws;
+  ws.ptr = at(0x40000000);
+  ws.bytes = ws_bytes;
+  try {
+    gemm(nullptr, at(0x10000000), lda, at(0x20000000), ldb, b_nk, false, at(0x30000000), N, M, N, K, GemmEpilogue(), ws, ev);
+  } catch (const Error& e) {
+    printf("M=%d N=%d K=%d %s: %s\n", M, N, K, b_nk ? "NK" : "KN", e.what());
+    return e.code;
+  }
+  return MFT_OK;
+}
+
+bool expect(bool ok, const char* what) {
+  if (!ok) printf("FAILED: %s\n", what);
+  return ok;
+}
+
+// Reductions too deep for one 32-bit buffer offset, whose slices are not: the
+// plan splits every tile, whatever the tile count is a multiple of.
+bool deep() {
+  bool ok = true;
+  struct Shape {
+    int M, N, K;
+    bool b_nk;
+    int64_t lda, ldb;
+    int slices;
+  };
+  const Shape shapes[] = {
+      {1024, 4096, 262144, false, 262144, 4096, 2},  // dlogits·E of a 4096-wide model: 256 tiles of 128×128
+      {768, 8192, 200000, false, 200000, 8192, 2},   // whole rounds of 64-row tiles, a round and a half of 128×128
+      {1100, 4352, 262144, false, 262144, 4352, 2},  // not a multiple
+      {64, 64, 8350000, true, 8350000, 8350000, 4},  // rows so long that A's and B's first 128 leave little for K
+  };
+  for (const Shape& s : shapes) {
+    const size_t ws = (size_t)s.slices * s.M * s.N * sizeof(float);
+    ok &= expect(status_of(s.M, s.N, s.K, s.b_nk, s.lda, s.ldb, ws + 256) == MFT_EHIP, "a deep reduction with room for its slices");
+    ok &= expect(status_of(s.M, s.N, s.K, s.b_nk, s.lda, s.ldb, 0) == MFT_EINVAL, "a deep reduction without a workspace");
+  }
+  return ok;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const char* mode = argc > 1 ? argv[1] : "";
+  bool ok = false;
+  if (!strcmp(mode, "deep")) ok = deep();
+  puts(ok ? "OK" : "FAILED");
+  return ok ? 0 : 1;
+}
