@@ -478,6 +478,12 @@ thread_local const KernelEvents* t_gemm_events = nullptr;
 thread_local hipEvent_t t_tail_start = nullptr, t_tail_stop = nullptr;
 namespace {
 
+// The timing events of the launches in a scope; none are left behind by one that throws.
+struct GemmEventScope {
+  explicit GemmEventScope(const KernelEvents* ev) { t_gemm_events = ev; }
+  ~GemmEventScope() { t_gemm_events = nullptr; }
+};
+
 // After the main launch: the split-K reduction with the epilogue (and the
 // row norm, fused into it where splitk_norm can), or the row norm alone.
 void gemm_finish(hipStream_t s, int splits, bool dispatch_events, const KernelEvents* ev, const float* partial,
@@ -655,6 +661,7 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
     pl = {bm, bn, sp, (int)(cdiv(M, bm) * cdiv(N, bn)), 0};
   MFT_CHECK_ARG(!ep.stats || (pl.bn == 128 && pl.splits == 1 && pl.tail_splits <= 1),
                 "row statistics need whole 128-wide tiles");
+  MFT_CHECK_ARG(gemm_x_depth(pl, p) <= k_max, "GEMM operand too large for 32-bit buffer offsets");
   static const bool log_plans = getenv("MFT_GEMM_PLAN_LOG") != nullptr;  // tuning hook: print each launch's plan
   if (log_plans)
     fprintf(stderr, "gemm %d,%d,%d:%d,%d,%d full=%d tail=%d norm=%d\n", M, N, K, pl.bm, pl.bn, pl.splits, pl.full,
@@ -672,10 +679,10 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
     tev.start = ev->tail_start;
     tev.stop = ev->tail_stop;
   }
-  t_gemm_events = dispatch_events ? ev : nullptr;
-  MFT_CHECK_ARG(gemm_x_depth(pl, p) <= k_max, "GEMM operand too large for 32-bit buffer offsets");
-  gemm_x_launch(s, p, pl, b_nk, b_f16, wsp, tev.start ? &tev : nullptr);
-  t_gemm_events = nullptr;
+  {
+    const GemmEventScope scope(dispatch_events ? ev : nullptr);
+    gemm_x_launch(s, p, pl, b_nk, b_f16, wsp, tev.start ? &tev : nullptr);
+  }
   if (ev && ev->stop && !dispatch_events) MFT_HIP(hipEventRecord(ev->stop, s));
 
   gemm_finish(s, p.partial ? p.tail_splits : 1, dispatch_events, ev, wsp, M, N, C, ldc, ep, nm);
@@ -738,11 +745,12 @@ void gemm_h(hipStream_t s, const float* A, int64_t lda, const float* inv_s, cons
   if (ev) MFT_HIP(hipStreamIsCapturing(s, &cap));
   const bool dispatch_events = ev && ev->start && ev->stop && cap == hipStreamCaptureStatusNone;
   if (ev && ev->start && !dispatch_events) MFT_HIP(hipEventRecord(ev->start, s));
-  t_gemm_events = dispatch_events ? ev : nullptr;
-  if (pl.bm == 128) launch_h<128, 128>(s, p, b_nk, splits);
-  else if (pl.bn == 128) launch_h<64, 128>(s, p, b_nk, splits);
-  else launch_h<64, 64>(s, p, b_nk, splits);
-  t_gemm_events = nullptr;
+  {
+    const GemmEventScope scope(dispatch_events ? ev : nullptr);
+    if (pl.bm == 128) launch_h<128, 128>(s, p, b_nk, splits);
+    else if (pl.bn == 128) launch_h<64, 128>(s, p, b_nk, splits);
+    else launch_h<64, 64>(s, p, b_nk, splits);
+  }
   if (ev && ev->stop && !dispatch_events) MFT_HIP(hipEventRecord(ev->stop, s));
   gemm_finish(s, splits, dispatch_events, ev, ws.ptr, M, N, C, ldc, ep, nm);
 }
@@ -797,11 +805,12 @@ bool gemm_h_segments(hipStream_t s, const float* A, int64_t lda, const float* in
   if (ev) MFT_HIP(hipStreamIsCapturing(s, &cap));
   const bool dispatch_events = ev && ev->start && ev->stop && cap == hipStreamCaptureStatusNone;
   if (ev && ev->start && !dispatch_events) MFT_HIP(hipEventRecord(ev->start, s));
-  t_gemm_events = dispatch_events ? ev : nullptr;
-  if (pl.bm == 128) launch_h<128, 128>(s, p, b_nk, 1);
-  else if (pl.bn == 128) launch_h<64, 128>(s, p, b_nk, 1);
-  else launch_h<64, 64>(s, p, b_nk, 1);
-  t_gemm_events = nullptr;
+  {
+    const GemmEventScope scope(dispatch_events ? ev : nullptr);
+    if (pl.bm == 128) launch_h<128, 128>(s, p, b_nk, 1);
+    else if (pl.bn == 128) launch_h<64, 128>(s, p, b_nk, 1);
+    else launch_h<64, 64>(s, p, b_nk, 1);
+  }
   if (ev && ev->stop && !dispatch_events) MFT_HIP(hipEventRecord(ev->stop, s));
   return true;
 }
@@ -858,11 +867,12 @@ void gemm_h_ksegments(hipStream_t s, const float* A, int64_t lda, const GemmHKSe
   if (ev) MFT_HIP(hipStreamIsCapturing(s, &cap));
   const bool dispatch_events = ev && ev->start && ev->stop && cap == hipStreamCaptureStatusNone;
   if (ev && ev->start && !dispatch_events) MFT_HIP(hipEventRecord(ev->start, s));
-  t_gemm_events = dispatch_events ? ev : nullptr;
-  if (pl.bm == 128) launch_h<128, 128>(s, p, true, splits);
-  else if (pl.bn == 128) launch_h<64, 128>(s, p, true, splits);
-  else launch_h<64, 64>(s, p, true, splits);
-  t_gemm_events = nullptr;
+  {
+    const GemmEventScope scope(dispatch_events ? ev : nullptr);
+    if (pl.bm == 128) launch_h<128, 128>(s, p, true, splits);
+    else if (pl.bn == 128) launch_h<64, 128>(s, p, true, splits);
+    else launch_h<64, 64>(s, p, true, splits);
+  }
   if (ev && ev->stop && !dispatch_events) MFT_HIP(hipEventRecord(ev->stop, s));
   gemm_finish(s, splits, dispatch_events, ev, ws.ptr, M, N, C, ldc, ep, nm);
 }

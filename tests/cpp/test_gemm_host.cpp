@@ -55,12 +55,22 @@ bool deep() {
   return ok;
 }
 
+// A call refused for its size leaves the caller's events as they were.
+bool timing() {
+  KernelEvents ev;
+  ev.start = ev.stop = ev.tail_start = ev.tail_stop = reinterpret_cast<hipEvent_t>(at(0x50000000));
+  bool ok = expect(status_of(64, 640, 1 << 20, false, 1 << 20, 1 << 20, 1 << 26, &ev) == MFT_EINVAL, "refused before any event is touched");
+  ok &= expect(!ev.tail_used, "no reduction was timed");
+  return ok;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const char* mode = argc > 1 ? argv[1] : "";
   bool ok = false;
   if (!strcmp(mode, "deep")) ok = deep();
+  if (!strcmp(mode, "timing")) ok = timing();
   puts(ok ? "OK" : "FAILED");
   return ok ? 0 : 1;
 }
