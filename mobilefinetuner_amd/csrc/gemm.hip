@@ -526,7 +526,7 @@ void launch_h_rank(hipStream_t s, GemmHParams& p, bool b_nk, int splits) {
   p.tiles_m = (int)cdiv(p.M, BM);
   p.tiles_n = (int)cdiv(p.N, BN);
   const dim3 grid = xcd_grid(p, splits), block(256);
-  p.out_vec = out_vec(p);
+  if (p.nseg <= 1) p.out_vec = out_vec(p);  // gemm_h_segments looks at every segment
   static const int pipe = [] {  // tuning hook: MFT_GEMMH_PIPE = 2 or 3 register staging sets
     const char* e = getenv("MFT_GEMMH_PIPE");
     return e && atoi(e) == 2 ? 2 : 3;
@@ -755,6 +755,12 @@ void gemm_h(hipStream_t s, const float* A, int64_t lda, const float* inv_s, cons
   gemm_finish(s, splits, dispatch_events, ev, ws.ptr, M, N, C, ldc, ep, nm);
 }
 
+bool segments_out_vec(const GemmHSegmentArg* seg, int nseg) {
+  bool vec = true;
+  for (int g = 0; g < nseg; ++g) vec = vec && seg[g].ldc % 4 == 0 && ((uintptr_t)seg[g].C & 15) == 0;
+  return vec;
+}
+
 bool gemm_h_segments(hipStream_t s, const float* A, int64_t lda, const float* inv_s, bool b_nk,
                      const GemmHSegmentArg* seg, int nseg, int M, int K, const GemmEpilogue& ep,
                      const KernelEvents* ev) {
@@ -793,6 +799,7 @@ bool gemm_h_segments(hipStream_t s, const float* A, int64_t lda, const float* in
   p.partial = nullptr;
   p.k_chunk = K;
   p.nseg = nseg;
+  p.out_vec = segments_out_vec(seg, nseg);
   for (int g = 0, n0 = 0; g < nseg; n0 += seg[g].N, ++g) {
     p.seg[g] = GemmHSegment{n0, seg[g].B, seg[g].ldb, seg[g].C, seg[g].ldc, seg[g].P, seg[g].Q};
     MFT_CHECK_ARG((b_nk ? (int64_t)pl.bn * seg[g].ldb + K : (int64_t)K * seg[g].ldb + pl.bn) * 2 < (int64_t(1) << 32),

@@ -220,6 +220,9 @@ int out_vec(const Params& p) {
                              (uintptr_t)p.ep.gelu_grad_of) & 15) == 0;
 }
 
+// The same for a column-segmented launch, whose tiles store to their own segment's C.
+bool segments_out_vec(const GemmHSegmentArg* seg, int nseg);
+
 // Launch of the GEMM kernel proper.  With timing events set, the dispatch
 // itself records them (hipExtLaunchKernel: the timestamps bracket the
 // kernel's execution), so timing adds no event packets to the stream and the

@@ -1,9 +1,11 @@
-// test_gemm_host.cpp — host side of the fp32 GEMMs, without a GPU: what
-// gemm() refuses and accepts.  An accepted call gets as far as its launch,
+// test_gemm_host.cpp — host side of the GEMMs, without a GPU: what
+// gemm() refuses and accepts, and launch rules.  An accepted call gets as far as its launch,
 // which fails here for want of a device (MFT_EHIP); a refused one throws
 // MFT_EINVAL before.  The operands are addresses that nothing reads.
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
+#include <utility>
 
 #include "gemm_common.h"
 
@@ -64,6 +66,25 @@ bool timing() {
   return ok;
 }
 
+// 16-byte output rows of a column-segmented launch: every segment's C and
+// pitch count, not the first one's.
+bool segments() {
+  auto vec = [](std::initializer_list<std::pair<uintptr_t, int64_t>> segs) {
+    GemmHSegmentArg a[3] = {};
+    int n = 0;
+    for (const auto& s : segs) {
+      a[n].C = at(s.first);
+      a[n++].ldc = s.second;
+    }
+    return segments_out_vec(a, n);
+  };
+  bool ok = expect(vec({{0x1000, 64}, {0x2000, 128}, {0x3010, 68}}), "aligned segments");
+  ok &= expect(!vec({{0x1000, 64}, {0x2004, 64}}), "a second segment off by four bytes");
+  ok &= expect(!vec({{0x1000, 64}, {0x2000, 64}, {0x3000, 65}}), "an odd pitch of the third");
+  ok &= expect(!vec({{0x1008, 64}, {0x2000, 64}}), "a first segment off by eight bytes");
+  return ok;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -71,6 +92,7 @@ int main(int argc, char** argv) {
   bool ok = false;
   if (!strcmp(mode, "deep")) ok = deep();
   if (!strcmp(mode, "timing")) ok = timing();
+  if (!strcmp(mode, "segments")) ok = segments();
   puts(ok ? "OK" : "FAILED");
   return ok ? 0 : 1;
 }

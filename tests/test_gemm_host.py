@@ -1,5 +1,5 @@
-"""Host side of the fp32 GEMMs on a machine without a GPU: which calls are
-refused (before anything is launched) and which get as far as their launch."""
+"""Host side of the GEMMs on a machine without a GPU: which calls are
+refused (before anything is launched) and which get as far as their launch; launch rules."""
 import os
 import subprocess
 
@@ -9,7 +9,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BIN = os.path.join(ROOT, "tests", "cpp", "bin", "test_gemm_host")
 
 
-@pytest.mark.parametrize("mode", ["deep", "timing"])
+@pytest.mark.parametrize("mode", ["deep", "timing", "segments"])
 def test_gemm_host(mode):
     assert os.path.exists(BIN), "tests/cpp/bin/test_gemm_host missing: run __graft_entry__.build()"
     # no visible device, also where there is one: the operands are no memory
