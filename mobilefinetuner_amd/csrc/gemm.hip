@@ -4,7 +4,7 @@
 //
 // gemm(): fp32 operands (or fp16 B of a shape the fp16 kernel does not take)
 // on the bf16 matrix cores, every fp32 value as three bf16 terms
-// (gemm_x.hip).  gemm_h(): fp16 B on the fp16 matrix cores, the fp32 operand
+// (gemm_x.hip), or, small products, on the fp32 matrix cores.  gemm_h(): fp16 B on the fp16 matrix cores, the fp32 operand
 // as two fp16 terms with a row scale.  Both fuse bias, the rank-r LoRA term
 // scale·P[M,r]·Q, a residual add and accumulation into C; split-K partials
 // are summed with the epilogue (and a row norm) by a second launch.
@@ -45,6 +45,235 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
       }
     }
   }
+}
+
+// ---- small fp32 products -------------------------------------------------------
+// C = A·op(B) on the fp32 matrix cores for products of few tiles (plan_gemm_x
+// chooses; both sides' times stand there).  gemm_x_kernel's panel step is a
+// chain of splitting instructions, 0.42 µs however small the tile; here it is
+// 16 MFMAs a wave, 0.21 µs of the matrix core, and 0.31 with the barrier and
+// the LDS reads that nothing hides at one workgroup a CU.  Half the tile, so
+// that small outputs reach more CUs.
+// Workgroup tile 32×64, four waves as 2×2, each owning 16×32 outputs as two
+// v_mfma_f32_16x16x4_f32 tiles; K in panels of 32.  Lane (i, g) supplies
+// A[row i][k g] and B[k g][col i] and holds D[row 4g+v][col i]; over four
+// consecutive MFMAs lane group g takes k = 4g..4g+3 of a 16-wide k block, so
+// an A or [N,K] B fragment is one 128-bit LDS read; with B as [K,N] the
+// wave's two column tiles interleave (tile b holds columns 2i + b) and one
+// 64-bit read a k gives a lane its B values of both.
+//
+// Every k step of two panels has accumulators of its own (sixteen sets of 8
+// registers, added pairwise at the end): no MFMA waits for the one before it,
+// and a chain holds K/16 products, so that from K = 256 on the sums are as
+// close to 64 bits as gemm_x_kernel's.
+//
+// Panel entry j lives in LDS stage j % 3 and is stored two steps before it is
+// multiplied, so that in step j every wave already holds the fragments of the
+// first k block of entry j+1; global loads run four entries ahead through two
+// register sets.  One barrier a step.  The loop runs two steps per iteration:
+// an odd panel count starts with an entry of zeros, and loads past the last
+// panel re-read it.  TAIL: K not a multiple of 32, or fp16 B; elements of the
+// last panel at k ≥ K are zeroed at the store.
+template <bool B_NK, bool B_F16, bool RANK, bool TAIL>
+__global__ __launch_bounds__(256) void gemm_s_kernel(GemmParams p) {
+  constexpr int BM = 32, BN = 64, BK = 32;
+  constexpr int PA = BK + 4;
+  // [K,N] B: 4·PB ≡ 32 (mod 64) puts lane groups g and g+1 of a 64-bit
+  // fragment read in disjoint LDS bank halves
+  constexpr int PB = B_NK ? BK + 4 : BN + 8;
+  constexpr int A_STAGE = BM * PA, STAGE = A_STAGE + (B_NK ? BN : BK) * PB;
+  constexpr int N_LD = 3;  // 16-byte chunks of a panel per thread: one of A, two of B
+  constexpr int BES = B_F16 ? 2 : 4;
+  __shared__ __attribute__((aligned(16))) float smem[3 * STAGE];
+
+  int tile, split;
+  float* raw_tile;
+  if (!tile_slice<BM, BN>(p, tile, split, raw_tile)) return;
+  const int m0 = tile % p.tiles_m * BM, n0 = tile / p.tiles_m * BN;
+  const int kbeg = split * p.k_chunk;
+  const int klen = tile < p.full_tiles ? p.K : min(p.K - kbeg, p.k_chunk);
+  const int nk = (klen + BK - 1) / BK, odd = nk & 1;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave & 1) * 16, wn = (wave >> 1) * 32;
+  const int li = lane & 15, lg = lane >> 4;
+
+  floatx4 acc[16][2];
+#pragma unroll
+  for (int t = 0; t < 16; ++t)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[t][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // buffer resources based at the tile's first row / column of its K-slice
+  const __amdgpu_buffer_rsrc_t rsa = buf_rsrc(p.A + (int64_t)m0 * p.lda + kbeg);
+  const __amdgpu_buffer_rsrc_t rsb =
+      buf_rsrc(static_cast<const char*>(p.B) + (B_NK ? (int64_t)n0 * p.ldb + kbeg : (int64_t)kbeg * p.ldb + n0) * BES);
+  const int a_row = tid / 8, kq = tid % 8 * 4;  // of [rows][32] chunks
+  const uint32_t a_off = (uint32_t)(((int64_t)(min(m0 + a_row, p.M - 1) - m0) * p.lda + kq) * 4);
+  uint32_t b_off[2];
+  int b_lds[2];  // LDS offsets (floats) within a stage
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    if constexpr (B_NK) {
+      const int row = a_row + 32 * it;
+      b_off[it] = (uint32_t)(((int64_t)(min(n0 + row, p.N - 1) - n0) * p.ldb + kq) * BES);
+      b_lds[it] = A_STAGE + row * PB + kq;
+    } else {
+      const int k = tid / 16 + 16 * it, nq = tid % 16 * 4;
+      b_off[it] = (uint32_t)(((int64_t)k * p.ldb + (n0 + nq < p.N ? nq : 0)) * BES);
+      b_lds[it] = A_STAGE + k * PB + nq;
+    }
+  }
+
+  floatx4 rs[2][N_LD];  // register staging sets
+  // entry j holds panel j − odd, clamped to the slice's
+  auto kof = [&](int j) { return min(max(j - odd, 0), nk - 1) * BK; };
+  // TAIL: chunks at k ≥ klen re-read the row's first of the panel, rows at
+  // k ≥ klen the panel's first row
+  auto gload = [&](auto sc, int j) {
+    constexpr int S = decltype(sc)::value;
+    const int kc = kof(j);
+    const uint32_t kback = TAIL && kc + kq >= klen ? (uint32_t)kq : 0u;
+    rs[S][0] = buf_load4(rsa, a_off - kback * 4u, (uint32_t)kc * 4u);
+    const uint32_t boff = (uint32_t)((B_NK ? (int64_t)kc : (int64_t)kc * p.ldb) * BES);
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int k = tid / 16 + 16 * it;
+      const uint32_t back = B_NK ? kback * BES : TAIL && kc + k >= klen ? (uint32_t)((int64_t)k * p.ldb) * BES : 0u;
+      if constexpr (B_F16) rs[S][1 + it] = stash_f16(buf_load2u(rsb, b_off[it] - back, boff));
+      else rs[S][1 + it] = buf_load4(rsb, b_off[it] - back, boff);
+    }
+  };
+  auto lstore = [&](auto sc, int stage, int j) {
+    constexpr int S = decltype(sc)::value;
+    float* st = smem + stage * STAGE;
+#pragma unroll
+    for (int it = 0; it < N_LD; ++it) {
+      floatx4 v = rs[S][it];
+      if (B_F16 && it > 0) v = unstash_f16(v);
+      if (TAIL) {  // without a branch, which would end the schedule of the step
+        const bool row = !B_NK && it > 0;  // the chunk lies along N
+        const int k = kof(j) + (row ? tid / 16 + 16 * (it - 1) : kq);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = k + (row ? 0 : e) < klen ? v[e] : 0.f;
+      }
+      *reinterpret_cast<floatx4*>(st + (it == 0 ? a_row * PA + kq : b_lds[it - 1])) = v;
+    }
+  };
+  struct Frags {
+    floatx4 a, b[2];
+  };
+  auto read_frags = [&](Frags& f, int stage, int kb) {
+    const float* as = smem + stage * STAGE;
+    const float* bs = as + A_STAGE;
+    f.a = *reinterpret_cast<const floatx4*>(as + (wm + li) * PA + kb + 4 * lg);
+    if constexpr (B_NK) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) f.b[b] = *reinterpret_cast<const floatx4*>(bs + (wn + 16 * b + li) * PB + kb + 4 * lg);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float2 v = *reinterpret_cast<const float2*>(bs + (kb + 4 * lg + t) * PB + wn + 2 * li);
+        f.b[0][t] = v.x;
+        f.b[1][t] = v.y;
+      }
+    }
+  };
+  auto mfmas = [&](const Frags& f, auto sc, auto qc) {
+    constexpr int T = 8 * decltype(sc)::value + 4 * decltype(qc)::value;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        acc[T + t][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[t], f.b[b][t], acc[T + t][b], 0, 0, 0);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+
+  constexpr int N_RD = 1 + (B_NK ? 2 : 4);  // LDS read instructions per read_frags
+  Frags F[2];
+  int s_cur = 0, s_nxt = 1, s_st = 2;  // stages of entries j, j+1, j+2 (wave-uniform)
+  auto step = [&](auto sc, int j) {
+    read_frags(F[1], s_cur, 16);
+    mfmas(F[0], sc, I0{});
+    read_frags(F[0], s_nxt, 0);  // entry j+1, visible since the last barrier
+    lstore(sc, s_st, j + 2);     // loaded two steps ago
+    gload(sc, j + 4);            // into the same register set
+    mfmas(F[1], sc, I1{});
+    __builtin_amdgcn_sched_group_barrier(0x100, N_RD, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, N_RD, 0);
+#pragma unroll
+    for (int i = 0; i < N_LD; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < N_LD; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 8 - 2 * N_LD, 0);
+    __syncthreads();
+    const int t = s_cur;
+    s_cur = s_nxt;
+    s_nxt = s_st;
+    s_st = t;
+  };
+  gload(I0{}, 0);
+  gload(I1{}, 1);
+  if (odd) {  // the entry of zeros
+    for (int i = tid; i < STAGE / 4; i += 256) reinterpret_cast<floatx4*>(smem)[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  } else {
+    lstore(I0{}, 0, 0);
+  }
+  lstore(I1{}, 1, 1);
+  gload(I0{}, 2);
+  gload(I1{}, 3);
+  __syncthreads();
+  read_frags(F[0], 0, 0);
+  for (int j = 0; j < nk + odd; j += 2) {
+    step(I0{}, j);
+    step(I1{}, j + 1);
+  }
+#pragma unroll
+  for (int o = 8; o >= 1; o /= 2)
+#pragma unroll
+    for (int t = 0; t < o; ++t)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[t][b] += acc[t + o][b];
+
+  // Rank-r LoRA term: one more K panel of depth r, staged in the ring's LDS
+  // after the last step's barrier; split 0 only.
+  if (RANK && split == 0) {
+    const int r = p.ep.r, rp = (r + 3) & ~3, pr = rp + 1;
+    float* Ps = smem;
+    float* Qs = smem + BM * pr;
+    for (int i = tid; i < BM * rp; i += 256) {
+      const int row = i / rp, j = i % rp, m = m0 + row;
+      Ps[row * pr + j] = (m < p.M && j < r) ? p.ep.P[(int64_t)m * r + j] : 0.f;
+    }
+    for (int i = tid; i < BN * rp; i += 256) {
+      const int col = i / rp, j = i % rp, n = n0 + col;
+      Qs[col * pr + j] = (n < p.N && j < r) ? p.ep.lscale * p.ep.Q[(int64_t)n * p.ep.qsn + (int64_t)j * p.ep.qsj] : 0.f;
+    }
+    __syncthreads();
+    for (int t = 0; t < rp / 4; ++t) {
+      const float fp = Ps[(wm + li) * pr + 4 * t + lg];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const float fq = Qs[(wn + (B_NK ? 16 * b + li : 2 * li + b)) * pr + 4 * t + lg];
+        acc[0][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fp, fq, acc[0][b], 0, 0, 0);
+      }
+    }
+  }
+  tile_out<BM, BN, 3 * STAGE * 4>(p, smem, m0, n0, split, [&](auto&& put) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) put(wm + 4 * lg + v, wn + (B_NK ? 16 * b + li : 2 * li + b), acc[0][b][v]);
+  }, raw_tile);
 }
 
 // ---- fp16 matrix-core path ---------------------------------------------------
@@ -520,6 +749,28 @@ void gemm_finish(hipStream_t s, int splits, bool dispatch_events, const KernelEv
 }
 
 
+// ---- small fp32 GEMM launch ----
+template <bool B_NK, bool B_F16, bool TAIL>
+void launch_s_rank(hipStream_t s, const GemmParams& p, dim3 grid) {
+  if (p.ep.P != nullptr) launch_gemm_kernel(gemm_s_kernel<B_NK, B_F16, true, TAIL>, grid, dim3(256), s, p);
+  else launch_gemm_kernel(gemm_s_kernel<B_NK, B_F16, false, TAIL>, grid, dim3(256), s, p);
+}
+}  // namespace
+void gemm_s_launch(hipStream_t s, const GemmParams& p, dim3 grid, bool b_nk, bool b_f16) {
+  if (b_f16) {
+    if (b_nk) launch_s_rank<true, true, true>(s, p, grid);
+    else launch_s_rank<false, true, true>(s, p, grid);
+  } else if (p.K % 32 == 0) {
+    if (b_nk) launch_s_rank<true, false, false>(s, p, grid);
+    else launch_s_rank<false, false, false>(s, p, grid);
+  } else {
+    if (b_nk) launch_s_rank<true, false, true>(s, p, grid);
+    else launch_s_rank<false, false, true>(s, p, grid);
+  }
+  MFT_LAUNCH_CHECK();
+}
+namespace {
+
 // ---- fp16 matrix-core GEMM launch ----
 template <int BM, int BN, bool RANK>
 void launch_h_rank(hipStream_t s, GemmHParams& p, bool b_nk, int splits) {
@@ -651,13 +902,13 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
   float* wsp = ws.ptr ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws.ptr) + skew) : nullptr;
   const size_t ws_bytes = ws.ptr && ws.bytes > skew ? ws.bytes - skew : 0;
   XPlan pl = plan_gemm_x(M, N, K, k_max, ws_bytes, nm != nullptr && N % 4 == 0 && N <= 4096 && ldc == N,
-                         ep.stats != nullptr);
+                         ep.stats != nullptr, b_f16 || K % 32 != 0);
   // Tuning hook: MFT_GEMM_PLAN="bm,bn,splits" (or per shape, "M,N,K:bm,bn,splits;...") forces tiles and a uniform split.
   static const char* forced_env = getenv("MFT_GEMM_PLAN");
   int bm = 0, bn = 0, sp = 0;
   if (!ep.stats && !b_f16 && forced_plan(forced_env, M, N, K, bm, bn, sp) &&
-      ((bm == 64 && bn == 64) || (bm == 64 && bn == 128) || (bm == 128 && bn == 128)) && sp >= 1 &&
-      (sp == 1 || (size_t)sp * M * N * sizeof(float) <= ws_bytes))
+      ((bm == 32 && bn == 64) || (bm == 64 && bn == 64) || (bm == 64 && bn == 128) || (bm == 128 && bn == 128)) &&
+      sp >= 1 && (sp == 1 || (size_t)sp * M * N * sizeof(float) <= ws_bytes))
     pl = {bm, bn, sp, (int)(cdiv(M, bm) * cdiv(N, bn)), 0};
   MFT_CHECK_ARG(!ep.stats || (pl.bn == 128 && pl.splits == 1 && pl.tail_splits <= 1),
                 "row statistics need whole 128-wide tiles");

@@ -91,6 +91,29 @@ __device__ __forceinline__ bool tile_of(const Params& p, int& tile, int& split) 
   return tile < tiles && split < p.splits;
 }
 
+// Workgroup → (tile, K-slice) of a GemmParams launch, and where a split
+// tile's raw sums go (null: the whole output or [slice][M][N] partials).
+// Workgroup L runs on XCD L % 8, each with its own L2: the whole tiles first,
+// contiguous runs of them (M-fastest) to an XCD, so that it reads whole column
+// bands of B; then the slices of the others, the slices of one K range
+// together, so that an XCD reads the A rows of few slices.
+template <int BM, int BN>
+__device__ __forceinline__ bool tile_slice(const GemmParams& p, int& tile, int& split, float*& raw_tile) {
+  const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8, rem = p.tiles_m * p.tiles_n - p.full_tiles;
+  raw_tile = nullptr;
+  split = 0;
+  if (idx < p.full_per_xcd) {
+    tile = xcd * p.full_per_xcd + idx;
+    return tile < p.full_tiles;
+  }
+  const int u = xcd * p.tail_per_xcd + idx - p.full_per_xcd;
+  if (u >= rem * p.tail_splits) return false;
+  split = u / rem;
+  tile = p.full_tiles + u % rem;
+  if (!p.partial) raw_tile = p.tail_out + ((int64_t)(u % rem) * p.tail_splits + split) * (min(BM, p.M) * BN);
+  return true;
+}
+
 // Bias, residual and β·C; the rank-r term is accumulated on the matrix
 // cores before the epilogue.
 __device__ __forceinline__ float epilogue_value(const GemmEpilogue& ep, float acc, int m, int n,
@@ -257,8 +280,8 @@ dim3 xcd_grid(Params& p, int splits) {
   return dim3((unsigned)(p.tiles_per_xcd * 8), 1);
 }
 
-// gemm_x.hip.  How gemm_x_launch runs C = A·op(B): tiles bm×bn of 64×64,
-// 64×128 or 128×128; with splits > 1 every tile in that many K-slices to
+// gemm_x.hip.  How gemm_x_launch runs C = A·op(B): tiles bm×bn of 32×64
+// (gemm_s_kernel), 64×64, 64×128 or 128×128 (gemm_x_kernel); with splits > 1 every tile in that many K-slices to
 // [slice][M][N] partials in ws, which the caller reduces; else the first
 // `full` tiles whole and the others in tail_splits slices, summed by a second
 // launch.
@@ -267,11 +290,13 @@ struct XPlan {
 };
 // norm: a row norm of the finished output follows (it rides in the
 // reduction of a uniform split); stats: 128-wide tiles, none split.
-// k_max: the deepest K-slice a tile may take.
-XPlan plan_gemm_x(int M, int N, int K, int64_t k_max, size_t ws_bytes, bool norm, bool stats);
+// k_max: the deepest K-slice a tile may take; tail: K not in whole panels, or fp16 B.
+XPlan plan_gemm_x(int M, int N, int K, int64_t k_max, size_t ws_bytes, bool norm, bool stats, bool tail);
 int gemm_x_depth(const XPlan& pl, const GemmParams& p);  // the deepest K-slice of a plan
 void gemm_x_launch(hipStream_t s, GemmParams& p, const XPlan& pl, bool b_nk, bool b_f16, float* ws,
                    const KernelEvents* tail_ev);
+// gemm.hip: gemm_s_kernel on a grid of tile_slice.
+void gemm_s_launch(hipStream_t s, const GemmParams& p, dim3 grid, bool b_nk, bool b_f16);
 
 }  // namespace mft
 #endif

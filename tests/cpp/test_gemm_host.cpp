@@ -85,6 +85,20 @@ bool segments() {
   return ok;
 }
 
+// Which products the 32×64 fp32 tiles take: at most a round of them, K from
+// 256 on, and no row statistics.
+bool small() {
+  auto bm = [](int M, int N, int K, bool stats = false) {
+    return plan_gemm_x(M, N, K, int64_t(1) << 28, size_t(64) << 20, false, stats, K % 32 != 0).bm;
+  };
+  bool ok = expect(bm(512, 768, 768) == 32 && bm(16, 256, 256) == 32 && bm(1024, 512, 512) == 32 && bm(300, 300, 300) == 32,
+                   "small products");
+  ok &= expect(bm(256, 256, 255) == 64 && bm(8, 64, 64) == 64, "K below 256");
+  ok &= expect(bm(1024, 640, 640) != 32 && bm(512, 3072, 768) != 32 && bm(1024, 4864, 896) != 32, "more than a round of tiles");
+  ok &= expect(bm(128, 1024, 512, true) == 128, "row statistics");
+  return ok;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -93,6 +107,7 @@ int main(int argc, char** argv) {
   if (!strcmp(mode, "deep")) ok = deep();
   if (!strcmp(mode, "timing")) ok = timing();
   if (!strcmp(mode, "segments")) ok = segments();
+  if (!strcmp(mode, "small")) ok = small();
   puts(ok ? "OK" : "FAILED");
   return ok ? 0 : 1;
 }

@@ -9,7 +9,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BIN = os.path.join(ROOT, "tests", "cpp", "bin", "test_gemm_host")
 
 
-@pytest.mark.parametrize("mode", ["deep", "timing", "segments"])
+@pytest.mark.parametrize("mode", ["deep", "timing", "segments", "small"])
 def test_gemm_host(mode):
     assert os.path.exists(BIN), "tests/cpp/bin/test_gemm_host missing: run __graft_entry__.build()"
     # no visible device, also where there is one: the operands are no memory

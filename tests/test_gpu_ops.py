@@ -329,6 +329,61 @@ def test_fp32_linear_tiny_against_large(K, same_sign):
         assert np.all(np.abs(y16 - ref16) <= b16), (xe, we, np.max(np.abs(y16 - ref16) / b16))
 
 
+# Edges of the 32×64 tiles of small products (K >= 256): one row, a row and a
+# column past a tile, panels of odd and even count, K tails, ragged
+# widths, a whole round of tiles, slices of few rows.
+SMALL_SHAPES = [(1, 256, 4, 0), (31, 256, 64, 4), (33, 260, 68, 8), (32, 288, 128, 32), (65, 284, 36, 16), (300, 300, 300, 8),
+                (512, 768, 768, 8), (19, 3976, 1068, 8), (19, 1068, 3976, 0), (40, 1000, 640, 0)]
+
+
+# fp16 W where the fp16 matrix cores do not take it
+SMALL_CASES = [(*s, w16) for s in SMALL_SHAPES for w16 in (False, True) if not w16 or s[1] % 32 or s[2] % 32]
+
+
+@pytest.mark.parametrize("M,K,N,r,w16", SMALL_CASES)
+def test_small_linear(M, K, N, r, w16):
+    """Forward with bias, residual and rank-r term and dX added to an old one,
+    against 64 bits.  Bound: sixteen chains of K/16 additions, the sums of the
+    chains, the rank-r chain and the epilogue's additions, each off by at most
+    2^-23 of the sum of magnitudes; the rank-r term counts twice, its first
+    factor being a rounded sum itself."""
+    print(f"small linear M={M} K={K} N={N} r={r} w16={w16}", flush=True)
+    x, dy, W, b, res, old = rn(M, K), rn(M, N), rn(K, N, std=0.05), rn(N), rn(M, N), rn(M, K)
+    W = W.astype(np.float16) if w16 else W
+    A, B = (rn(r, K, std=1 / 8), rn(N, r, std=0.02)) if r else (None, None)
+    d = lambda a: a.astype(np.float64)  # noqa: E731
+    def check(got, terms, rank, depth):
+        # depth: additions of the longest chain
+        ref = sum(p @ q if q is not None else p for p, q in terms)
+        mag = sum(np.abs(p) @ np.abs(q) if q is not None else np.abs(p) for p, q in terms)
+        if r:
+            mag = mag + 2 * 2.0 * np.abs(rank[0]) @ np.abs(rank[1]) @ np.abs(rank[2])
+            ref = ref + 2.0 * rank[0] @ rank[1] @ rank[2]
+        assert np.all(np.abs(h(got) - ref) <= (depth / 16 + 16 + r) * 2.0 ** -23 * mag)
+    lora_f = (d(x), d(A).T, d(B).T) if r else None
+    lora_b = (d(dy), d(B), d(A)) if r else None
+    gA, gB = (g(A), g(B)) if r else (None, None)
+    y, xa = ops.lora_linear_fwd(g(x), g(W), g(b), gA, gB, 2.0, resid=g(res))
+    check(y, [(d(x), d(W)), (d(b)[None, :], None), (d(res), None)], lora_f, K)
+    dx = g(old)
+    ops.lora_linear_bwd(g(dy), g(x), g(W), gA, gB, xa, 2.0, dx=dx, dx_accumulate=True)
+    check(dx, [(d(dy), d(W).T), (d(old), None)], lora_b, N)
+
+
+@pytest.mark.parametrize("M,K,N", [(256, 256, 256), (512, 768, 768), (64, 512, 512), (100, 1000, 640), (256, 128, 256)])
+def test_small_linear_error(M, K, N):
+    """The error of small products over a whole output.  Sixteen chains of
+    K/16 products and four levels of their sums make, for operands of either
+    sign, an rms of 2.8e-8·sqrt(K/32 + 4) of the result (one rounding in each
+    addition); the three-term kernel that takes K < 256 has less.  Held to
+    twice that, which one lost bf16 product of it (4e-6) is far from."""
+    x, dy, W = rn(M, K), rn(M, N), rn(K, N, std=0.05)
+    y, _ = ops.lora_linear_fwd(g(x), g(W), None, None, None, 1.0)
+    assert rel_err(h(y), x.astype(np.float64) @ W.astype(np.float64)) < 5.6e-8 * math.sqrt(K / 32 + 4)
+    dx, _, _ = ops.lora_linear_bwd(g(dy), None, g(W), None, None, None, 1.0)
+    assert rel_err(h(dx), dy.astype(np.float64) @ W.astype(np.float64).T) < 5.6e-8 * math.sqrt(N / 32 + 4)
+
+
 @pytest.mark.parametrize("M,K,r", [(1, 8, 32), (511, 2048, 8), (513, 2052, 4), (1025, 2048, 8), (1027, 2300, 4),
                                    (70, 2048, 16), (33, 516, 32)])
 def test_rank_projection_row_groups(M, K, r):
