@@ -172,10 +172,9 @@ def test_lora_linear_fp16_k_tail_takes_widened_path():
 
 def test_lm_head_fp16_vocab_gemms():
     """Gemma-3 1B's LM head with the tied embedding E [V, d] stored as fp16
-    (config 5): logits = h·Eᵀ runs the 128×128 kernel with an [N, K] fp16
-    operand widened in the tile load (8192 tiles at M = 512, V = 262144), and
-    dH = dlogits·E reduces over the whole vocabulary (K = 262144, split 16
-    ways).  Both against the oracle (BLAS-backed GEMMs) on the same fp16
+    (config 5), on the fp16 matrix cores: logits = h·Eᵀ with an [N, K] operand
+    (V = 262144), and dH = dlogits·E, which reduces over the whole vocabulary
+    (K = 262144, split).  Both against the oracle (BLAS-backed GEMMs) on the same fp16
     values, at the fp32 bar."""
     M, d, V = 512, 1152, 262144
     print(f"lm head fp16 M={M} d={d} V={V}", flush=True)
@@ -198,20 +197,20 @@ def test_lm_head_fp16_vocab_gemms():
 
 
 PIPE_SHAPES = [
-    (512, 1024, 4096, False),  # 64x64 tiles, 32 whole panels
-    (512, 1024, 1024, False),  # 32x64 tiles
+    (512, 1024, 4096, False),  # 32 whole panels
+    (512, 1024, 1024, False),  # 256 tiles of 32x64
     (200, 96, 300, False),     # three panels (odd count), ragged M and N
     (512, 4096, 1024, False),  # split-K: whole panels in every split
-    (128, 1152, 1024, True),   # fp16 W widened in the pipelined tile load
+    (128, 1152, 1024, True),   # fp16 W on the fp16 matrix cores
 ]
 
 
 @pytest.mark.parametrize("M,K,N,f16", PIPE_SHAPES)
 def test_plain_linear_pipelined(M, K, N, f16):
-    """Linears without a rank-r panel whose K splits into whole 32-deep panels:
-    dX (W as the [N,K] operand of dY·Wᵀ) runs the three-stage pipelined GEMM,
-    the forward (W as [K,N]) the two-stage one; both against the oracle,
-    including an odd panel count, split-K and fp16 W."""
+    """Linears without a rank-r panel whose K splits into whole 32-deep panels,
+    in the pipelined GEMMs: dX (W as the [N,K] operand of dY·Wᵀ) and the
+    forward (W as [K,N]) against the oracle, including an odd panel count,
+    split-K and fp16 W."""
     print(f"pipelined gemm M={M} K={K} N={N} f16={f16}", flush=True)
     x, dy, b = rn(M, K), rn(M, N), rn(N)
     W = rn(K, N, std=0.03)
@@ -269,6 +268,50 @@ def test_fp32_linear_on_bf16_matrix_cores(M, K, N):
     if N % 4 == 0:
         dx, _, _ = ops.lora_linear_bwd(g(dy), g(x), g(W), None, None, None, 1.0)
         within(h(dx), dy, W.T, 0.0)
+
+
+# The forward ([K,N] W) and dX ([N,K] W) of each: whole 64×64 tiles (256×224),
+# 64×64 with a split remainder and 64×128 all split (512×768×2304 and its dX),
+# K tails on 64×64 and 64×128, whole and split, 128×128 whole (1024×640×4096),
+# all split (its dX) and with a split remainder and a K tail (1024×1096×4868).
+ERROR_SHAPES = [(256, 224, 200), (512, 768, 2304), (512, 2304, 768), (130, 1028, 1100), (300, 2052, 2044),
+                (700, 612, 2300), (1024, 640, 4096), (1024, 4096, 640), (1024, 1096, 4868), (2000, 224, 2048)]
+
+
+@pytest.mark.parametrize("M,K,N", ERROR_SHAPES)
+def test_fp32_linear_error(M, K, N):
+    """The error over a whole output, which the elementwise bound above leaves
+    far below itself where K is deep.  An accumulation every 16 products, cut
+    off at 2^-23 of the sum so far, makes an rms of about 6e-9·sqrt(K) of the
+    result for operands of either sign; held to twice that.  One lost product
+    of the six shows at 2.4e-6 (hi·lo), 2.8e-6 (mid·mid) or more at any depth."""
+    print(f"split gemm error M={M} K={K} N={N}", flush=True)
+    x, dy, W = rn(M, K), rn(M, N), rn(K, N, std=0.05)
+    y, _ = ops.lora_linear_fwd(g(x), g(W), None, None, None, 1.0)
+    assert rel_err(h(y), x.astype(np.float64) @ W.astype(np.float64)) < 4e-8 + 1.2e-8 * math.sqrt(K)
+    dx, _, _ = ops.lora_linear_bwd(g(dy), None, g(W), None, None, None, 1.0)
+    assert rel_err(h(dx), dy.astype(np.float64) @ W.astype(np.float64).T) < 4e-8 + 1.2e-8 * math.sqrt(N)
+
+
+@pytest.mark.parametrize("M,K,N,r", [(130, 1028, 1101, 8), (512, 3072, 771, 0), (600, 2304, 904, 4)])
+def test_split_tile_epilogue(M, K, N, r):
+    """The sums of split tiles with every term of the epilogue: bias, residual
+    and rank-r panel in the forward, an old dX added to, at odd widths (element
+    by element) and whole ones (16 bytes at a time).  Each term is as large as
+    the product, so that one left out or added per slice shows.  The GELU terms
+    are covered by the full-size GPT-2 step (512×768×3072 and its dX)."""
+    print(f"split tile epilogue M={M} K={K} N={N} r={r}", flush=True)
+    x, W, b, res = rn(M, K), rn(K, N, std=1 / math.sqrt(K)), rn(N), rn(M, N)
+    A, B = (rn(r, K, std=1 / math.sqrt(K)), rn(N, r, std=1 / math.sqrt(r))) if r else (None, None)
+    d = lambda a: a.astype(np.float64)  # noqa: E731
+    y, _ = ops.lora_linear_fwd(g(x), g(W), g(b), g(A) if r else None, g(B) if r else None, 2.0, resid=g(res))
+    lora = 2.0 * d(x) @ d(A).T @ d(B).T if r else 0.0
+    assert rel_err(h(y), d(x) @ d(W) + d(b) + d(res) + lora) < 4e-8 + 1.2e-8 * math.sqrt(K)
+    # dX of the transposed layer: the same reduction into an output N wide
+    old = rn(M, N)
+    dx = g(old)
+    ops.lora_linear_bwd(g(x), None, g(W.T.copy()), None, None, None, 1.0, dx=dx, dx_accumulate=True)
+    assert rel_err(h(dx), d(x) @ d(W) + d(old)) < 4e-8 + 1.2e-8 * math.sqrt(K)
 
 
 @pytest.mark.parametrize("M,K,N", [(70, 68, 96), (256, 1024, 256)])
