@@ -107,13 +107,14 @@ __global__ __launch_bounds__(1024) void ce_count_kernel(const int32_t* __restric
 // in flight per thread, each group of 4·U values folded into the thread's
 // running (max, Σ) pair with one rescale, and re-read by the gradient sweep,
 // which writes dlogits in place.
-// Wide rows (H = 16, L = 8, 96 Ki values held) are bound by HBM: the held
-// values, the second reading of the rest and the dlogits bypass the caches
-// (non-temporal), which leaves them to the values still to be read again.
-// 1024 rows of 262144 values: 592 µs with 64 Ki held and plain accesses, 555
-// with LDS, 516 with non-temporal stores, 459 with the loads too (4.7 TB/s of
-// the 8·V bytes a row; a copy reaches 4.8); 151936: 326 → 245.  Rows that fit
-// in registers measured slower with non-temporal loads (42 → 46 µs).
+// Wide rows (H = 16, L = 8, 96 Ki values held) are bound by HBM: the values
+// held in registers, the second reading of the rest and the dlogits bypass
+// the caches (non-temporal), which leaves them to the values still to be read
+// again (those held in LDS are read with plain loads).  1024 rows of 262144
+// values: 592 µs with 64 Ki held and plain accesses, 555 with LDS, 516 with
+// non-temporal stores, 459 with the loads too (4.7 TB/s of the 8·V bytes a
+// row; a copy of that size reaches 5.0); 151936: 326 → 245.  Rows that fit in
+// registers measured slower with non-temporal loads (42 → 46 µs).
 // The micro-batch's target count is formed in every workgroup beside the
 // row's statistics (workgroup 0 stores it in *cnt and raises *bad), or, with
 // `counted`, read from *cnt where ce_count_kernel stored it.

@@ -372,8 +372,31 @@ struct GemmHParams {
   GemmHKSegment kseg[kMaxGemmHSegments];
 };
 
-// C = diag(inv_s)·(hi + lo)·op(B) (+ the rank-r panel and epilogue of
-// gemm_p_kernel), hi/lo the fp16 split of diag(s)·A made while A's fp32
+// Workgroup → (tile, split) of a 1-D grid.  Workgroup L runs on XCD L % 8
+// (round-robin dispatch), each XCD with its own L2.  With s ≤ 8 splits, the
+// s K-slices take 8/s XCDs each and their tiles are cut into contiguous
+// ranges among those XCDs, M-fastest, so an XCD reads whole column bands of
+// B and the A rows of only its own K-slice (a split-K launch that spread
+// every slice over every XCD would fetch the whole of A into each of the 8
+// L2s).  With `spread` (used for s > 8) every K-slice covers all 8 XCDs.
+// Host side: tiles_per_xcd = ceil(tiles / (8/s)), or ceil(tiles/8) spread.
+__device__ __forceinline__ bool tile_of(const GemmHParams& p, int& tile, int& split) {
+  const int L = blockIdx.x, xcd = L % 8, idx = L / 8;
+  const int tiles = p.tiles_m * p.tiles_n;
+  if (p.spread) {
+    const int per = 8 * p.tiles_per_xcd, r = L % per;
+    split = L / per;
+    tile = (r % 8) * p.tiles_per_xcd + r / 8;
+  } else {  // s ≤ 8
+    const int g = 8 / p.splits;  // XCDs per split
+    split = xcd / g;
+    tile = (xcd % g) * p.tiles_per_xcd + idx;
+  }
+  return tile < tiles && split < p.splits;
+}
+
+// C = diag(inv_s)·(hi + lo)·op(B) (+ a rank-r panel on the fp32 matrix cores,
+// and tile_out's epilogue), hi/lo the fp16 split of diag(s)·A made while A's fp32
 // panel is staged into LDS.  Workgroup tile BM×BN, four waves as 2×2, each
 // owning (BM/2)×(BN/2) outputs as 16×16 tiles; K in panels of 32 (one
 // v_mfma_f32_16x16x32_f16 k-block: lane l holds row l%16, k 8(l/16)..+7 of
@@ -383,10 +406,10 @@ struct GemmHParams {
 // 4a+e of every 16-lane group element e of the 8-byte rows addressed by
 // lanes a, a+4, a+8, a+12 — lanes addressing rows k..k+3 at columns
 // n0 + 4·(0..3) give each lane four consecutive k of its own column, so W
-// needs no transposed copy.  Pipeline as in gemm_p_kernel: a three-stage
-// LDS ring stored two steps ahead, global loads four steps ahead in two
-// register sets, fragments of the next stage read at the top of each step,
-// one barrier per step.  Row pitches: 40 halves (A, [N,K] B: 16-byte
+// needs no transposed copy.  Pipeline: a three-stage LDS ring stored two
+// steps ahead, global loads PIPE + 2 steps ahead in PIPE register sets,
+// fragments of the next stage read at the top of each step, one barrier per
+// step.  Row pitches: 40 halves (A, [N,K] B: 16-byte
 // fragment reads conflict-free over 8 lanes), BN + 16 halves (k-major B:
 // the four rows of a 16-lane transposed read fall in disjoint banks).
 template <int BM, int BN, bool B_NK, bool RANK, int PIPE>
@@ -772,6 +795,23 @@ void gemm_s_launch(hipStream_t s, const GemmParams& p, dim3 grid, bool b_nk, boo
 namespace {
 
 // ---- fp16 matrix-core GEMM launch ----
+dim3 xcd_grid(GemmHParams& p, int splits) {
+  static const int spread = [] {  // tuning hook: MFT_GEMM_SPREAD=1 spreads every K-slice over all XCDs
+    const char* e = getenv("MFT_GEMM_SPREAD");
+    return e ? atoi(e) : 0;
+  }();
+  const int tiles = p.tiles_m * p.tiles_n;
+  p.splits = splits;
+  // up to eight slices have XCDs of their own (1024×1152×6912 60 µs, spread
+  // 65; the other fp16 layer shapes level); beyond there is none left for each
+  p.spread = spread || splits > 8;
+  if (p.spread) {
+    p.tiles_per_xcd = (int)cdiv(tiles, 8);
+    return dim3((unsigned)(p.tiles_per_xcd * 8 * splits), 1);
+  }
+  p.tiles_per_xcd = (int)cdiv(tiles, 8 / splits);
+  return dim3((unsigned)(p.tiles_per_xcd * 8), 1);
+}
 template <int BM, int BN, bool RANK>
 void launch_h_rank(hipStream_t s, GemmHParams& p, bool b_nk, int splits) {
   p.tiles_m = (int)cdiv(p.M, BM);

@@ -67,30 +67,6 @@ __device__ __forceinline__ float2 row_stats64(const float* row) {
   return make_float2(ml, s0 + s1);
 }
 
-// Workgroup → (tile, split) of a 1-D grid.  Workgroup L runs on XCD L % 8
-// (round-robin dispatch), each XCD with its own L2.  With s ≤ 8 splits, the
-// s K-slices take 8/s XCDs each and their tiles are cut into contiguous
-// ranges among those XCDs, M-fastest, so an XCD reads whole column bands of
-// B and the A rows of only its own K-slice (a split-K launch that spread
-// every slice over every XCD would fetch the whole of A into each of the 8
-// L2s).  With `spread` (used for s > 8) every K-slice covers all 8 XCDs.
-// Host side: tiles_per_xcd = ceil(tiles / (8/s)), or ceil(tiles/8) spread.
-template <class Params>
-__device__ __forceinline__ bool tile_of(const Params& p, int& tile, int& split) {
-  const int L = blockIdx.x, xcd = L % 8, idx = L / 8;
-  const int tiles = p.tiles_m * p.tiles_n;
-  if (p.spread) {
-    const int per = 8 * p.tiles_per_xcd, r = L % per;
-    split = L / per;
-    tile = (r % 8) * p.tiles_per_xcd + r / 8;
-  } else {  // s ≤ 8
-    const int g = 8 / p.splits;  // XCDs per split
-    split = xcd / g;
-    tile = (xcd % g) * p.tiles_per_xcd + idx;
-  }
-  return tile < tiles && split < p.splits;
-}
-
 // Workgroup → (tile, K-slice) of a GemmParams launch, and where a split
 // tile's raw sums go (null: the whole output or [slice][M][N] partials).
 // Workgroup L runs on XCD L % 8, each with its own L2: the whole tiles first,
@@ -163,8 +139,8 @@ __device__ __forceinline__ void epilogue_store4(const GemmEpilogue& ep, floatx4 
   }
 }
 
-// Output of a 2×2-wave tile of 16×16 accumulators (gemm_h_kernel,
-// gemm_x_kernel): partials of a split K, or the epilogue.  The tile goes
+// Output of a 2×2-wave tile (gemm_s_kernel, gemm_h_kernel, gemm_x_kernel):
+// partials of a split K, or the epilogue.  The tile goes
 // through the idle LDS ring (row pitch BN + 4 floats), so that a thread
 // handles 16-byte runs of whole rows: loads and stores of 256 or 512
 // contiguous bytes, and one small loop for the whole tile.  Straight from
@@ -258,26 +234,6 @@ void launch_gemm_kernel(Kern kernel, dim3 grid, dim3 block, hipStream_t s, const
     hipExtLaunchKernelGGL(kernel, grid, block, 0, s, t_gemm_events->start, t_gemm_events->stop, 0, p);
   else
     hipLaunchKernelGGL(kernel, grid, block, 0, s, p);
-}
-
-template <class Params>
-dim3 xcd_grid(Params& p, int splits) {
-  static const int spread = [] {  // tuning hook: MFT_GEMM_SPREAD=1 spreads every K-slice over all XCDs
-    const char* e = getenv("MFT_GEMM_SPREAD");
-    return e ? atoi(e) : 0;
-  }();
-  const int tiles = p.tiles_m * p.tiles_n;
-  p.splits = splits;
-  // vocabulary-deep reductions (the LM head's dH, 16 splits) measured 1.4%
-  // faster with every slice over all XCDs; layer GEMMs keep one K-slice per
-  // XCD group (43% less L2 fetch on GPT-2 small, same time)
-  p.spread = spread || splits > 8;
-  if (p.spread) {
-    p.tiles_per_xcd = (int)cdiv(tiles, 8);
-    return dim3((unsigned)(p.tiles_per_xcd * 8 * splits), 1);
-  }
-  p.tiles_per_xcd = (int)cdiv(tiles, 8 / splits);
-  return dim3((unsigned)(p.tiles_per_xcd * 8), 1);
 }
 
 // gemm_x.hip.  How gemm_x_launch runs C = A·op(B): tiles bm×bn of 32×64
