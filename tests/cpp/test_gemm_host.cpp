@@ -85,9 +85,17 @@ bool segments() {
   return ok;
 }
 
-// Which products the 32×64 fp32 tiles take: at most a round of them, K from
-// 256 on, and no row statistics.
+// Which products the 32×64 fp32 tiles take: at most a round of them, slices of
+// K from 256 on, and no row statistics.
 bool small() {
+  for (int M : {8, 32, 100, 300})
+    for (int N : {36, 256, 1068})
+      for (int K : {260, 480, 1040, 2048, 3976, 65536}) {
+        const XPlan p = plan_gemm_x(M, N, K, int64_t(1) << 28, size_t(64) << 20, false, false, K % 32 != 0);
+        GemmParams g{};
+        g.K = K;
+        if (p.bm == 32 && !expect(gemm_x_depth(p, g) >= 256, "slices of small tiles")) return false;
+      }
   auto bm = [](int M, int N, int K, bool stats = false) {
     return plan_gemm_x(M, N, K, int64_t(1) << 28, size_t(64) << 20, false, stats, K % 32 != 0).bm;
   };
