@@ -302,8 +302,7 @@ def main():
         kname = ("linear-layer GEMMs (gemm_h_kernel: fp16 W on fp16 MFMA, fp32 operand as hi+lo fp16, "
                  "rank-r panel on fp32 MFMA; fwd + dX) with their split-K reductions" if mc.w_fp16 else
                  "linear-layer GEMMs (gemm_x_kernel: fp32 operands as three bf16 terms each, six bf16 MFMA "
-                 "products; the smallest gemm_s_kernel on fp32 MFMA; fwd + dX, merged LoRA weights) with their "
-                 "split-K reductions")
+                 "products; fwd + dX, merged LoRA weights) with their split-K reductions")
         result["roofline"] = {
             "kernel": kname, "bound": "mfma",
             "achieved": round(ach, 2), "peak": round(peak_mm, 1), "unit": "TFLOP/s",

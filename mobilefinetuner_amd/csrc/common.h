@@ -160,6 +160,12 @@ struct GemmEpilogue {
   //                 of the activation's input from that of its output.
   float* gelu_out = nullptr;
   const float* gelu_grad_of = nullptr;
+  // The operators' linears: small products may take gemm_s_kernel's tiles.  The
+  // step engine's passes keep gemm_x_kernel throughout: after Adam's first
+  // steps, which follow a gradient's sign, other sums at the rounding floor
+  // move weights the other way, and a resumed run is to go on as it would have
+  // with the version before.
+  bool small_tiles = false;
   // LM head (128×128 plan only): per row and 64-column block of C, the
   // base-2 softmax statistics (max of C·log2e, Σ 2^(C·log2e − max)) of the
   // stored values, at stats[row·stats_ld + n/64]; the cross-entropy then

@@ -4,7 +4,7 @@
 //
 // gemm(): fp32 operands (or fp16 B of a shape the fp16 kernel does not take)
 // on the bf16 matrix cores, every fp32 value as three bf16 terms
-// (gemm_x.hip), or, small products, on the fp32 matrix cores.  gemm_h(): fp16 B on the fp16 matrix cores, the fp32 operand
+// (gemm_x.hip), or, small products of the operators, on the fp32 matrix cores.  gemm_h(): fp16 B on the fp16 matrix cores, the fp32 operand
 // as two fp16 terms with a row scale.  Both fuse bias, the rank-r LoRA term
 // scale·P[M,r]·Q, a residual add and accumulation into C; split-K partials
 // are summed with the epilogue (and a row norm) by a second launch.
@@ -942,7 +942,7 @@ void gemm(hipStream_t s, const float* A, int64_t lda, const void* B, int64_t ldb
   float* wsp = ws.ptr ? reinterpret_cast<float*>(reinterpret_cast<char*>(ws.ptr) + skew) : nullptr;
   const size_t ws_bytes = ws.ptr && ws.bytes > skew ? ws.bytes - skew : 0;
   XPlan pl = plan_gemm_x(M, N, K, k_max, ws_bytes, nm != nullptr && N % 4 == 0 && N <= 4096 && ldc == N,
-                         ep.stats != nullptr, b_f16 || K % 32 != 0);
+                         ep.stats != nullptr, ep.small_tiles, b_f16 || K % 32 != 0);
   // Tuning hook: MFT_GEMM_PLAN="bm,bn,splits" (or per shape, "M,N,K:bm,bn,splits;...") forces tiles and a uniform split.
   static const char* forced_env = getenv("MFT_GEMM_PLAN");
   int bm = 0, bn = 0, sp = 0;

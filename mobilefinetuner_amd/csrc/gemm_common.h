@@ -246,8 +246,9 @@ struct XPlan {
 };
 // norm: a row norm of the finished output follows (it rides in the
 // reduction of a uniform split); stats: 128-wide tiles, none split.
-// k_max: the deepest K-slice a tile may take; tail: K not in whole panels, or fp16 B.
-XPlan plan_gemm_x(int M, int N, int K, int64_t k_max, size_t ws_bytes, bool norm, bool stats, bool tail);
+// small: 32×64 tiles too; k_max: the deepest K-slice a tile may take; tail: K
+// not in whole panels, or fp16 B.
+XPlan plan_gemm_x(int M, int N, int K, int64_t k_max, size_t ws_bytes, bool norm, bool stats, bool small, bool tail);
 int gemm_x_depth(const XPlan& pl, const GemmParams& p);  // the deepest K-slice of a plan
 void gemm_x_launch(hipStream_t s, GemmParams& p, const XPlan& pl, bool b_nk, bool b_f16, float* ws,
                    const KernelEvents* tail_ev);

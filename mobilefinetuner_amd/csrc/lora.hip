@@ -28,6 +28,7 @@ void lora_linear_fwd(hipStream_t s, const float* x, int64_t M, int64_t K,
   GemmEpilogue ep;
   ep.bias = bias;
   ep.resid = resid;
+  ep.small_tiles = true;
   if (A && B && r > 0) {
     MFT_CHECK_ARG(xa != nullptr, "xa buffer required when LoRA is active");
     rank_proj(s, x, K, A, /*ysk=*/1, /*ysj=*/K, (int)M, (int)K, r, xa);
@@ -62,6 +63,7 @@ void lora_linear_bwd(hipStream_t s, const float* dy, const float* x,
   if (dx) {
     GemmEpilogue ep;
     ep.beta = dx_accumulate ? 1.f : 0.f;
+    ep.small_tiles = true;
     if (lora) {
       ep.P = U;
       ep.Q = A;  // Q(n=k, j) = A[j, k]

@@ -91,19 +91,20 @@ bool small() {
   for (int M : {8, 32, 100, 300})
     for (int N : {36, 256, 1068})
       for (int K : {260, 480, 1040, 2048, 3976, 65536}) {
-        const XPlan p = plan_gemm_x(M, N, K, int64_t(1) << 28, size_t(64) << 20, false, false, K % 32 != 0);
+        const XPlan p = plan_gemm_x(M, N, K, int64_t(1) << 28, size_t(64) << 20, false, false, true, K % 32 != 0);
         GemmParams g{};
         g.K = K;
         if (p.bm == 32 && !expect(gemm_x_depth(p, g) >= 256, "slices of small tiles")) return false;
       }
-  auto bm = [](int M, int N, int K, bool stats = false) {
-    return plan_gemm_x(M, N, K, int64_t(1) << 28, size_t(64) << 20, false, stats, K % 32 != 0).bm;
+  auto bm = [](int M, int N, int K, bool stats = false, bool small = true) {
+    return plan_gemm_x(M, N, K, int64_t(1) << 28, size_t(64) << 20, false, stats, small, K % 32 != 0).bm;
   };
   bool ok = expect(bm(512, 768, 768) == 32 && bm(16, 256, 256) == 32 && bm(1024, 512, 512) == 32 && bm(300, 300, 300) == 32,
                    "small products");
   ok &= expect(bm(256, 256, 255) == 64 && bm(8, 64, 64) == 64, "K below 256");
   ok &= expect(bm(1024, 640, 640) != 32 && bm(512, 3072, 768) != 32 && bm(1024, 4864, 896) != 32, "more than a round of tiles");
   ok &= expect(bm(128, 1024, 512, true) == 128, "row statistics");
+  ok &= expect(bm(512, 768, 768, false, false) == 64 && bm(16, 256, 256, false, false) == 64, "the engine's products");
   return ok;
 }
 
